@@ -12,7 +12,8 @@
 // with d_t = (t/9 - 1, (t/3)%3 - 1, t%3 - 1) and periodic wrap.  Weights are
 // FP32 (o, i, 27).  An output of the data kernels is one chain of FMAs over
 // channels and, within them, taps.  The weight kernel sums chunks of the points,
-// then the chunks, in a fixed order without atomics.  All FP32 with FMA.
+// each as 256 chains of FMAs, then the chunks, in a fixed order without atomics.
+// All FP32 with FMA.
 #include <algorithm>
 
 #include "common.hpp"
@@ -467,325 +468,212 @@ static int launch_conv(const ConvDims& d, const float* x, const float* w, const 
 }
 
 // ------------------------------------------------------------------ //
-// Weight gradient: a product over the points, on v_mfma_f32_16x16x4_f32.  A
-// (16 channels x 4 points) is the array read in place, u; B (4 points x 16
-// columns) is the one read at the taps, s: a column is a channel of s at a
-// row (dz, dy) of taps, and the row's three taps are the same six values
-// shifted, so that four points of a lane cost one 16-byte read of u, 24 bytes
-// of s a block of columns and 12 products a block.  u is gy and s is x (SWAP =
-// false) or the other way round (taps mirrored), whichever leaves fewer
-// lanes idle: a column block holds 16 channels, or all nine rows of one
-// channel, or two blocks those of two or three.
-// A workgroup takes a chunk of the tiles of 8 x 8 x 2 points (x, y, z), MT blocks
-// of channels of u and one block of channels of s (NT column blocks); a wave
-// one block of u on 1 / WP of the tile's points.  The products of 16 points are
-// one chain from zero, added to the wave's sums (the error against 64 bits is
-// 0.5 to 0.9 of that of a thread's chain over every 256th point; chains over
-// all points of a wave had up to 2.2 of it).  The waves' sums meet in LDS, the
-// chunks' in wgrad_reduce_kernel, always in the same order.
-// Bound by the latency of a tile's loads and barriers with two workgroups a
-// CU, the matrix unit at 40 to 45% (23% of it at 16^3, where the partial sums'
-// 56 MB count).  Batch 8: 64^3 2 -> 16 130 us and 16 -> 1 90, 32^3 16 -> 32 110,
-// 32 -> 16 113, 16^3 32 -> 64 80 and 64 -> 32 73.  A workgroup a pair of channels
-// with all operands from memory took 603, 333, 1131, 1120, 636 and 631 us.
+// Weight gradient.  The B P points are cut into chunks, and a chunk's sum is
+// 256 chains of FMAs, chain r over the points r, r + 256, .. of the chunk, then
+// summed by halves (r and r + 128, r + 64, ..); the chunks are summed in order.
+// This order is kept for its bits: an optimiser step takes the weights from
+// them, and the next pass's results follow the weights.
+//
+// A thread carries a chain (workgroup: a chunk) of 9 taps, one dz, of OB outputs
+// and IB inputs: 72 chains in registers fed by 9 IB + OB loads, of which the
+// next point's are in flight.  A channel's base is uniform, so that a point
+// costs 33 instructions of index arithmetic for its 72 FMAs.  Bound by the
+// vector units and the loads' way through the L1 in about equal parts, three
+// workgroups a CU (two with 16 outputs a thread: no gain).  Batch 8: 64^3 2 ->
+// 16 130 us and 16 -> 1 167, 32^3 16 -> 32 217, 32 -> 16 212, 16^3 32 -> 64 and
+// 64 -> 32 120.  A workgroup a pair of channels took 609, 333, 1134, 1127, 637
+// and 633; products on the matrix units, in another order, 126, 85, 106, 108, 69
+// and 65.
 
-constexpr int kWTiles = 128;                 // points of a tile
-constexpr int kWU = kWTiles + 4;             // pitch of a channel of u
-constexpr long kWGroups = 512;               // workgroups wanted, two a CU
-constexpr int kWX = 12, kWS = 484;           // pitch of a row and of a channel of s
+constexpr int kWThreads = 256;
 
 struct WgradDims {
-    int B, Cu, Cs, D, H, W;
-    int cb;              // channels of s in a block
-    int nchunk, nub, nsb;   // chunks of tiles, blocks of u (16 MT) and of s (cb)
-    long ntiles, per;    // tiles in all, and of a chunk
+    int B, Cin, Cout, D, H, W;
+    int nchunk;
+    long chunk;          // points of a chunk
+    int sz, sy, sx;      // 256 points further along the grid
 };
 
-template <int MT, int NT, bool SWAP>
-__global__ __launch_bounds__(256, 2) void wgrad_kernel(const float* __restrict__ u,
-                                                       const float* __restrict__ s,
-                                                       float* __restrict__ part,
-                                                       float* __restrict__ partb, WgradDims d)
+// I: byte offsets within an array, 32 bits where they fit
+template <int OB, int IB, typename I>
+__global__ __launch_bounds__(kWThreads, 3) void wgrad_kernel(const float* __restrict__ x,
+                                                             const float* __restrict__ gy,
+                                                             float* __restrict__ part,
+                                                             float* __restrict__ partb,
+                                                             WgradDims d)
 {
-    constexpr int CS = NT == 9 ? 16 : (NT == 2 ? 3 : 1);
-    constexpr int WP = 4 / MT;
-    constexpr int NA = NT * 3 * 4 * 64;      // sums of a wave
-    constexpr int STAGE = CS * kWS + 16 * MT * kWU;
-    constexpr int LDS = WP > 1 && MT * NA > STAGE ? MT * NA : STAGE;
-    __shared__ __attribute__((aligned(16))) float lds[LDS];
-    __shared__ float bsum[4][16];
-    float* ss = lds;
-    float* us = lds + CS * kWS;
-
-    const long nwork = (long)d.nchunk * d.nub * d.nsb;
-    const long w = xcd_work_index(blockIdx.x, nwork);
+    constexpr int NV = 9 * OB * IB;          // chains, and those of the bias
+    __shared__ float red[2][NV + OB][64];
+    const int nob = (d.Cout + OB - 1) / OB, nib = (d.Cin + IB - 1) / IB;
+    const long w = xcd_work_index(blockIdx.x, (long)d.nchunk * 3 * nib * nob);
     if (w < 0) return;
-    const int blk = (int)(w % (d.nub * d.nsb)), chunk = (int)(w / (d.nub * d.nsb));
-    const int u0 = blk % d.nub * 16 * MT, s0 = blk / d.nub * d.cb;
-    const long t0 = chunk * d.per, t1 = min(d.ntiles, t0 + d.per);
-    const int ntx = (d.W + 7) / 8, nty = (d.H + 7) / 8, ntz = (d.D + 1) / 2;
+    const int o0 = (int)(w % nob) * OB;
+    long r = w / nob;
+    const int i0 = (int)(r % nib) * IB;
+    r /= nib;
+    const int dz = (int)(r % 3), chunk = (int)(r / 3);
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
     const long P = (long)d.D * d.H * d.W;
-    const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-    const int mt = wave % MT, pw = wave / MT;
-    const int g = lane / 16, n = lane % 16;
-
-    // staging: this thread's two points of s (tile with halo, 10 x 10 x 4)
-    // and point of u, all channels
-    float sr[CS][2], ur[8 * MT];
-    bool u_ok = false;
-    const int up = tid % kWTiles, uc = tid / kWTiles;
-    // the tile in flight: points, and the sample
-    int x0 = (int)(t0 % ntx) * 8, y0 = (int)(t0 / ntx % nty) * 8;
-    int z0 = (int)(t0 / ((long)ntx * nty) % ntz) * 2, b = (int)(t0 / ((long)ntx * nty * ntz));
-    auto advance = [&]() {
-        x0 += 8;
-        if (x0 >= d.W) x0 = 0, y0 += 8;
-        if (y0 >= d.H) y0 = 0, z0 += 2;
-        if (z0 >= d.D) z0 = 0, b++;
-    };
+    const long q0 = chunk * d.chunk, q1 = min((long)d.B * P, q0 + d.chunk);
+    // of the chains past the chunk: the last point, not used
+    const long q = min(q0 + tid, q1 - 1);
+    int left = q0 + tid < q1 ? (int)((q1 - q0 - tid + kWThreads - 1) / kWThreads) : 0;
+    int b = (int)(q / P), px, py, pz;
+    {
+        const int p = (int)(q % P);
+        px = p % d.W;
+        py = p / d.W % d.H;
+        pz = p / d.W / d.H;
+    }
+    auto at = [](const float* base, I byte) { return *(const float*)((const char*)base + byte); };
+    float xn[IB][9], gn[OB];
     auto load = [&]() {
-        const float* sb = s + (long)b * d.Cs * P;
-        unsigned off[2];
+        const I xb = (I)b * (I)(4 * P) * (I)d.Cin, gb = (I)b * (I)(4 * P) * (I)d.Cout;
+        const int z = wrapp(pz + dz - 1, d.D);
+        const int ry[3] = {wrapp(py - 1, d.H), py, wrapp(py + 1, d.H)};
+        const int cx[3] = {wrapp(px - 1, d.W), px, wrapp(px + 1, d.W)};
 #pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const int q = min(tid + 256 * e, 399);
-            const int gx = wrapm(x0 - 1 + q % 10, d.W);
-            const int gy = wrapm(y0 - 1 + q / 10 % 10, d.H);
-            const int gz = wrapm(z0 - 1 + q / 100, d.D);
-            off[e] = (gz * d.H + gy) * d.W + gx;
+        for (int t = 0; t < 9; t++) {
+            const I off = xb + 4 * (I)((z * d.H + ry[t / 3]) * d.W + cx[t % 3]);
+#pragma unroll
+            for (int i = 0; i < IB; i++) xn[i][t] = at(x + min(i0 + i, d.Cin - 1) * P, off);
         }
+        const I off = gb + 4 * (I)((pz * d.H + py) * d.W + px);
 #pragma unroll
-        for (int c = 0; c < CS; c++) {
-            const float* p = sb + min(s0 + c, d.Cs - 1) * P;
-#pragma unroll
-            for (int e = 0; e < 2; e++) sr[c][e] = p[off[e]];
-        }
-        const int gx = x0 + up % 8, gy = y0 + up / 8 % 8, gz = z0 + up / 64;
-        u_ok = gx < d.W && gy < d.H && gz < d.D;
-        const unsigned uo = u_ok ? (gz * d.H + gy) * d.W + gx : 0;
-        const float* ub = u + (long)b * d.Cu * P;
-#pragma unroll
-        for (int e = 0; e < 8 * MT; e++)
-            ur[e] = ub[min(u0 + uc + 2 * e, d.Cu - 1) * P + uo];
+        for (int o = 0; o < OB; o++) gn[o] = at(gy + min(o0 + o, d.Cout - 1) * P, off);
     };
-    // this lane's columns: their channel and row of taps in the tile of s
-    int sl[NT];
+    auto advance = [&]() {
+        px += d.sx;
+        if (px >= d.W) px -= d.W, py++;
+        py += d.sy;
+        if (py >= d.H) py -= d.H, pz++;
+        pz += d.sz;
+        while (pz >= d.D) pz -= d.D, b++;
+    };
+    float acc[NV + OB];
 #pragma unroll
-    for (int j = 0; j < NT; j++) {
-        const int col = 16 * j + n, r = col / d.cb, i = col % d.cb;
-        sl[j] = r < 9 ? i * kWS + (r / 3 * 10 + r % 3) * kWX : 0;   // idle past the ninth
-    }
-    f32x4 acc[NT][3];
-#pragma unroll
-    for (int j = 0; j < NT; j++)
-#pragma unroll
-        for (int dx = 0; dx < 3; dx++) acc[j][dx] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float accb = 0.f;   // sum of gy: of u's channel n, or of the column's (row 4)
-
+    for (int v = 0; v < NV + OB; v++) acc[v] = 0.f;
+    // the bias sums are those of one block of inputs and one dz
+    const bool bias = i0 == 0 && dz == 1;
     load();
-    for (long t = t0; t < t1; t++) {
-        lds_barrier();
+    while (left > 0) {
+        float xv[IB][9], g[OB];
 #pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const int q = tid + 256 * e;
-            if (q < 400)
+        for (int i = 0; i < IB; i++)
 #pragma unroll
-                for (int c = 0; c < CS; c++)
-                    ss[c * kWS + q / 10 * kWX + q % 10] = s0 + c < d.Cs ? sr[c][e] : 0.f;
-        }
+            for (int t = 0; t < 9; t++) xv[i][t] = xn[i][t];
 #pragma unroll
-        for (int e = 0; e < 8 * MT; e++) {
-            const int c = uc + 2 * e;
-            us[c * kWU + up] = u_ok && u0 + c < d.Cu ? ur[e] : 0.f;
-        }
-        const int xw = d.W - x0, yw = d.H - y0, zw = d.D - z0;   // what of the tile is in the grid
-        advance();
-        if (t + 1 < t1) load();
-        lds_barrier();
-        const bool whole = xw >= 8 && yw >= 8 && zw >= 2;
-#pragma unroll 1
-        for (int rr = pw; rr < 8; rr += WP) {
-            if (rr / 4 >= zw || rr % 4 * 2 >= yw) continue;
-            const int z = rr / 4, yy = rr % 4 * 2 + g / 2, xx = g % 2 * 4;
-            const float4 a4 = *(const float4*)(us + (16 * mt + n) * kWU + (z * 8 + yy) * 8 + xx);
-            const float av[4] = {a4.x, a4.y, a4.z, a4.w};
-            if (!SWAP) accb += (av[0] + av[1]) + (av[2] + av[3]);
-            const bool row_ok = yy < yw && z < zw;
+        for (int o = 0; o < OB; o++) g[o] = gn[o];
+        left--;
+        if (left > 0) advance();
+        load();                              // (past the last: the last again)
 #pragma unroll
-            for (int j = 0; j < NT; j++) {
-                const float* f = ss + sl[j] + (z * 10 + yy) * kWX + xx;
-                const float4 lo = *(const float4*)f;
-                const float2 hi = *(const float2*)(f + 4);
-                const float v[6] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y};
-                f32x4 run[3];
+        for (int i = 0; i < IB; i++)
 #pragma unroll
-                for (int dx = 0; dx < 3; dx++) run[dx] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < 9; t++)
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    // points outside the grid: zero times zero
-                    const bool ok = whole || (row_ok && xx + q < xw);
-                    if (SWAP && j == 0) accb += ok ? v[q + 1] : 0.f;
-#pragma unroll
-                    for (int dx = 0; dx < 3; dx++)
-                        run[dx] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                            av[q], ok ? v[q + dx] : 0.f, run[dx], 0, 0, 0);
+                for (int o = 0; o < OB; o++) {
+                    float& s = acc[(o * IB + i) * 9 + t];
+                    s = __builtin_fmaf(g[o], xv[i][t], s);
                 }
+        if (bias)
 #pragma unroll
-                for (int dx = 0; dx < 3; dx++) acc[j][dx] += run[dx];
-            }
-        }
+            for (int o = 0; o < OB; o++) acc[NV + o] += g[o];
     }
-    // the waves of a block of u, in order
-    accb += __shfl_xor(accb, 16);
-    accb += __shfl_xor(accb, 32);
-    if (g == 0) bsum[wave][n] = accb;
+    // chains r and r + 128, then r + 64, by waves; the rest by a thread a sum,
+    // which reads a row turned by its number so that no two share a bank
+    if (wave >= 2)
 #pragma unroll
-    for (int r = 1; r < WP; r++) {
-        __syncthreads();
-        if (pw == r) {
-#pragma unroll
-            for (int j = 0; j < NT; j++)
-#pragma unroll
-                for (int dx = 0; dx < 3; dx++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        lds[mt * NA + ((j * 3 + dx) * 4 + v) * 64 + lane] = acc[j][dx][v];
-        }
-        __syncthreads();
-        if (pw == 0) {
-#pragma unroll
-            for (int j = 0; j < NT; j++)
-#pragma unroll
-                for (int dx = 0; dx < 3; dx++)
-#pragma unroll
-                    for (int v = 0; v < 4; v++)
-                        acc[j][dx][v] += lds[mt * NA + ((j * 3 + dx) * 4 + v) * 64 + lane];
-        }
-    }
+        for (int v = 0; v < NV + OB; v++) red[wave - 2][v][lane] = acc[v];
     __syncthreads();
-    if (pw != 0) return;
-    float* dst = part + (((long)chunk * d.nub * d.nsb + blk) * MT + mt) * NA + lane;
+    if (wave < 2)
 #pragma unroll
-    for (int j = 0; j < NT; j++)
-#pragma unroll
-        for (int dx = 0; dx < 3; dx++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) dst[((j * 3 + dx) * 4 + v) * 64] = acc[j][dx][v];
-    // the sums of gy, from the workgroups of the first block of the other array
-    const int co = SWAP ? s0 + n - 4 * d.cb : u0 + 16 * mt + n;
-    const bool first = SWAP ? u0 == 0 && mt == 0 && n >= 4 * d.cb && n < 5 * d.cb : s0 == 0;
-    if (g == 0 && first && co < (SWAP ? d.Cs : d.Cu)) {
-        float sum = bsum[mt][n];
-#pragma unroll
-        for (int r = 1; r < WP; r++) sum += bsum[r * MT + mt][n];
-        partb[(long)chunk * (SWAP ? d.Cs : d.Cu) + co] = sum;
-    }
-}
-
-// gW and gb = sums over the chunks: 32 sums a workgroup, eight runs of chunks
-// each, then the runs in order
-template <int MT, int NT, bool SWAP>
-__global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restrict__ part,
-                                                           const float* __restrict__ partb,
-                                                           float* __restrict__ gW,
-                                                           float* __restrict__ gb, WgradDims d)
-{
-    constexpr int NA = NT * 3 * 4 * 64;
-    __shared__ float red[8][33];
-    const long nw = (long)d.nub * d.nsb * MT * NA;
-    const int nb = SWAP ? d.Cs : d.Cu;
-    const int c = threadIdx.x % 32, run = threadIdx.x / 32;
-    const long q = (long)blockIdx.x * 32 + c;
-    float sum = 0.f;
-    if (q < nw + nb) {
-        const float* p = q < nw ? part + q : partb + (q - nw);
-        const long step = q < nw ? nw : nb;
-#pragma unroll 8
-        for (int k = run; k < d.nchunk; k += 8) sum += p[k * step];
-    }
-    red[run][c] = sum;
+        for (int v = 0; v < NV + OB; v++) {
+            acc[v] += red[wave][v][lane];
+            if (wave == 1) red[1][v][lane] = acc[v];
+        }
     __syncthreads();
-    if (run || q >= nw + nb) return;
+    if (wave == 0)
 #pragma unroll
-    for (int r = 1; r < 8; r++) sum += red[r][c];
-    if (q >= nw) {
-        if (gb) gb[q - nw] = sum;
-        return;
+        for (int v = 0; v < NV + OB; v++) red[0][v][(lane + v) % 64] = acc[v] + red[1][v][lane];
+    __syncthreads();
+    if (tid >= NV + OB) return;
+    float sum[64];
+#pragma unroll
+    for (int k = 0; k < 64; k++) sum[k] = red[0][tid][(k + tid) % 64];
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1)
+#pragma unroll
+        for (int k = 0; k < s; k++) sum[k] += sum[k + s];
+    if (tid < NV) {
+        const int o = o0 + tid / (9 * IB), i = i0 + tid / 9 % IB;
+        if (o < d.Cout && i < d.Cin)
+            part[(((long)chunk * d.Cout + o) * d.Cin + i) * 27 + 9 * dz + tid % 9] = sum[0];
+    } else if (bias && o0 + tid - NV < d.Cout) {
+        partb[(long)chunk * d.Cout + o0 + tid - NV] = sum[0];
     }
-    const int lane = (int)(q % 64), v = (int)(q / 64 % 4), dx = (int)(q / 256 % 3);
-    const int j = (int)(q / 768 % NT);
-    const long um = q / NA;   // block of u within the block of s
-    const int mt = (int)(um % MT), blk = (int)(um / MT);
-    const int cu = blk % d.nub * 16 * MT + 16 * mt + 4 * (lane / 16) + v;
-    const int col = 16 * j + lane % 16, r = col / d.cb;
-    const int cs = blk / d.nub * d.cb + col % d.cb;
-    if (r >= 9 || cu >= d.Cu || cs >= d.Cs) return;
-    const int o = SWAP ? cs : cu, i = SWAP ? cu : cs, t = SWAP ? 26 - 3 * r - dx : 3 * r + dx;
-    gW[((long)o * (SWAP ? d.Cu : d.Cs) + i) * 27 + t] = sum;
 }
 
-static long wgrad_tiles(const ConvDims& c)
+// gW and gb = sums over the chunks, in order
+__global__ __launch_bounds__(64) void wgrad_reduce_kernel(const float* __restrict__ part,
+                                                          const float* __restrict__ partb,
+                                                          float* __restrict__ gW,
+                                                          float* __restrict__ gb, long n, int Cout,
+                                                          int nchunk)
 {
-    return (long)c.B * ((c.D + 1) / 2) * ((c.H + 7) / 8) * ((c.W + 7) / 8);
+    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n + (gb ? Cout : 0)) return;
+    const float* p = k < n ? part + k : partb + (k - n);
+    const long step = k < n ? n : Cout;
+    float s = 0.f;
+#pragma unroll 16
+    for (int c = 0; c < nchunk; c++) s += p[c * step];
+    if (k < n) gW[k] = s;
+    else gb[k - n] = s;
 }
 
-template <int MT, int NT, bool SWAP>
+// A block of outputs by one input; for one or two outputs one of them by a
+// block of inputs.
 static int launch_wgrad(const ConvDims& c, const float* x, const float* gy, float* gw, float* gb,
                         hipStream_t st)
 {
-    WgradDims d;
-    d.B = c.B;
-    d.Cu = SWAP ? c.Cin : c.Cout;
-    d.Cs = SWAP ? c.Cout : c.Cin;
-    d.D = c.D;
-    d.H = c.H;
-    d.W = c.W;
-    d.cb = NT == 9 ? 16 : d.Cs;
-    d.nub = (d.Cu + 16 * MT - 1) / (16 * MT);
-    d.nsb = (d.Cs + d.cb - 1) / d.cb;
-    d.ntiles = wgrad_tiles(c);
-    const long blocks = (long)d.nub * d.nsb;
-    d.nchunk = (int)std::max(1L, std::min(d.ntiles, kWGroups / blocks));
-    d.per = (d.ntiles + d.nchunk - 1) / d.nchunk;
-    d.nchunk = (int)((d.ntiles + d.per - 1) / d.per);
-    const long nw = blocks * MT * NT * 3 * 4 * 64;
+    // chunks of at least 4096 points, and so that a pair of channels and a
+    // chunk are about 2048 items
+    const long P = (long)c.D * c.H * c.W, npts = c.B * P, pairs = (long)c.Cout * c.Cin;
+    long nchunk = std::max(1L, std::min((2048 + pairs - 1) / pairs, npts / 4096));
+    WgradDims d = {c.B, c.Cin, c.Cout, c.D, c.H, c.W};
+    d.chunk = (npts + nchunk - 1) / nchunk;
+    nchunk = (npts + d.chunk - 1) / d.chunk;
+    d.nchunk = (int)nchunk;
+    d.sx = kWThreads % c.W;
+    d.sy = kWThreads / c.W % c.H;
+    d.sz = kWThreads / c.W / c.H;
+    const long n = pairs * 27;
     float* part = nullptr;
-    hipError_t e = hipMallocAsync((void**)&part, sizeof(float) * (nw + c.Cout) * d.nchunk, st);
+    hipError_t e = hipMallocAsync((void**)&part, sizeof(float) * (n + c.Cout) * nchunk, st);
     if (e != hipSuccess) {
         set_last_error(hipGetErrorString(e));
         return GPD_ERR_HIP;
     }
-    float* partb = part + nw * d.nchunk;
-    hipLaunchKernelGGL((wgrad_kernel<MT, NT, SWAP>), dim3(xcd_grid_size(blocks * d.nchunk)),
-                       dim3(256), 0, st, SWAP ? x : gy, SWAP ? gy : x, part, partb, d);
+    float* partb = part + n * nchunk;
+    const auto launch = [&](auto kernel, int ob, int ib) {
+        const long nwork = nchunk * 3 * ((c.Cin + ib - 1) / ib) * ((c.Cout + ob - 1) / ob);
+        hipLaunchKernelGGL(kernel, dim3(xcd_grid_size(nwork)), dim3(kWThreads), 0, st, x, gy, part,
+                           partb, d);
+    };
+    const bool fits = 4 * npts * std::max(c.Cin, c.Cout) < (1L << 32);
+    if (c.Cout <= 2)
+        fits ? launch(wgrad_kernel<1, 8, unsigned>, 1, 8) : launch(wgrad_kernel<1, 8, size_t>, 1, 8);
+    else
+        fits ? launch(wgrad_kernel<8, 1, unsigned>, 8, 1) : launch(wgrad_kernel<8, 1, size_t>, 8, 1);
     int rc = last_error_to_status(hipGetLastError());
     if (!rc) {
-        hipLaunchKernelGGL((wgrad_reduce_kernel<MT, NT, SWAP>),
-                           dim3((unsigned)((nw + c.Cout + 31) / 32)), dim3(256), 0, st, part,
-                           partb, gw, gb, d);
+        hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((unsigned)((n + c.Cout + 63) / 64)), dim3(64),
+                           0, st, part, partb, gw, gb, n, c.Cout, d.nchunk);
         rc = last_error_to_status(hipGetLastError());
     }
     (void)hipFreeAsync(part, st);
     return rc;
-}
-
-// s is the array of one to three channels where there is one.  With many
-// channels in both, a workgroup takes up to 64 of u (the staged points of s
-// serve them all), fewer where that would leave workgroups without a tile
-// (one sample of 4^3, 32 -> 64: 21 us with 16 channels, 39 with 64).
-static int dispatch_wgrad(const ConvDims& c, const float* x, const float* gy, float* gw,
-                          float* gb, hipStream_t st)
-{
-    if (c.Cin == 1) return launch_wgrad<1, 1, false>(c, x, gy, gw, gb, st);
-    if (c.Cout == 1) return launch_wgrad<1, 1, true>(c, x, gy, gw, gb, st);
-    if (c.Cin <= 3) return launch_wgrad<1, 2, false>(c, x, gy, gw, gb, st);
-    if (c.Cout <= 3) return launch_wgrad<1, 2, true>(c, x, gy, gw, gb, st);
-    const long work = wgrad_tiles(c) * ((c.Cin + 15) / 16);
-    if (c.Cout > 32 && work * ((c.Cout + 63) / 64) >= kWGroups)
-        return launch_wgrad<4, 9, false>(c, x, gy, gw, gb, st);
-    if (c.Cout > 16 && work * ((c.Cout + 31) / 32) >= kWGroups)
-        return launch_wgrad<2, 9, false>(c, x, gy, gw, gb, st);
-    return launch_wgrad<1, 9, false>(c, x, gy, gw, gb, st);
 }
 
 // leaky ReLU and its gradient (slope a for x < 0), elementwise
@@ -902,7 +790,7 @@ extern "C" int gpd_conv3d_backward_weight(int B, int Cin, int Cout, int D, int H
     GPD_REQUIRE((long)Cout * Cin <= (1L << 30), GPD_ERR_ARG, "too many channel pairs");
     ConvDims d = {B, Cin, Cout, D, H, W};
     hipStream_t st = (hipStream_t)stream;
-    return dispatch_wgrad(d, d_x, d_gy, d_gw, d_gb, st);
+    return launch_wgrad(d, d_x, d_gy, d_gw, d_gb, st);
 }
 
 extern "C" int gpd_leaky_relu(long n, float slope, const float* d_x, float* d_y, void* stream)
