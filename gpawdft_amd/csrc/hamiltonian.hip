@@ -96,14 +96,15 @@ __global__ void fill_zero_kernel(long n, T* __restrict__ p)
 // an event of one call, without timing
 struct Event {
     hipEvent_t e = nullptr;
-    hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming);
     ~Event()
     {
-        if (rc == hipSuccess) (void)hipEventDestroy(e);
+        if (e) (void)hipEventDestroy(e);
     }
     // `second` goes on after what `first` has now
     hipError_t order(hipStream_t first, hipStream_t second)
     {
+        if (first == second) return hipSuccess;
+        hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming);
         if (rc == hipSuccess) rc = hipEventRecord(e, first);
         return rc == hipSuccess ? hipStreamWaitEvent(second, e, 0) : rc;
     }
@@ -162,7 +163,6 @@ extern "C" int gpd_hamiltonian_apply_projected(gpd_operator* kin, gpd_lfc* lfc, 
 {
     GPD_REQUIRE(dtype == GPD_F64 || dtype == GPD_F32, GPD_ERR_ARG, "unknown dtype");
     GPD_REQUIRE(nb >= 0 && nP >= 0, GPD_ERR_ARG, "bad sizes");
-    GPD_REQUIRE(stream != side, GPD_ERR_ARG, "the second stream must be another one");
     if (nb == 0 && nP == 0) return GPD_OK;
     GPD_REQUIRE(kin && lfc && d_P && d_c && Mmax > 0 && nP / Mmax >= nb, GPD_ERR_ARG,
                 "bad projector arrays");

@@ -225,8 +225,8 @@ int gpd_lfc_destroy(gpd_lfc* lfc);
  * (GPD_F64, GPD_F32) in one call: P (nP values, at least nb rows of Mmax)
  * cleared and filled with the projections and c = P dH (the tables of
  * gpd_projector_coefs) on stream `side` while the stencil and v psi run on
- * `stream`, which then waits for it and adds the projector terms.  Not for
- * use under graph capture.                                              */
+ * `stream`, which then waits for it and adds the projector terms; one after
+ * the other where side is stream.  Not for use under graph capture.     */
 int gpd_hamiltonian_apply_projected(gpd_operator* kin, gpd_lfc* lfc, int dtype,
                                     long nb, const void* d_psi,
                                     const void* d_v, int Mmax, int natoms,
