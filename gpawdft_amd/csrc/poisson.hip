@@ -380,8 +380,11 @@ static int run_bottom(const VCycle& v)
 {
     size_t bytes = 0;
     for (int l = v.bottom; l <= v.levels; l++) bytes += 3 * sizeof(double) * grid_points(v.ops[l]);
+    // the process's attribute, always the same: another thread's call may come
+    // between this and the launch
     hipError_t e = hipFuncSetAttribute((const void*)poisson_bottom_kernel,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+                                       hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)kBottomBytes);
     if (e != hipSuccess) {
         set_last_error(hipGetErrorString(e));
         return GPD_ERR_HIP;
