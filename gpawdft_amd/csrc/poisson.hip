@@ -458,40 +458,50 @@ static int relax_tiles(const VCycle& v, int level, int sweeps, int launches, con
     return rc;
 }
 
+// The array that a level's sweeps may alternate with: its residual, which the
+// coarsest level has no use for otherwise and a caller need not keep for it.
+static double* second_array(const VCycle& v, int level)
+{
+    return level < v.levels || level == 0 ? v.residuals[level] : nullptr;
+}
+
 // Launches of `sweeps` Jacobi sweeps of the level, alternating between phi
-// and res.
+// and its second array.
 static int relax_launches(const VCycle& v, int level, int sweeps)
 {
     const int m = sweeps_per_launch(v, level);
     return m ? (sweeps + m - 1) / m : sweeps;
 }
 
-// Relaxation from the array `from` (phi or res) to phi; the other of the two
-// is its second array, so an odd number of launches that starts in phi is
+// Relaxation from the array `from` (phi or the second array) to phi; an odd
+// number of launches that starts in phi, or one without a second array, is
 // left to gpd_operator_relax and its copy (as are the calls it refuses).
 static int relax(const VCycle& v, int level, int sweeps, double* from)
 {
-    double* phi = v.phis[level];
-    if (sweeps > 0 && sweeps_per_launch(v, level)) {
+    double *phi = v.phis[level], *other = second_array(v, level);
+    if (other && sweeps > 0 && sweeps_per_launch(v, level)) {
         int launches = relax_launches(v, level, sweeps);
         if (from == phi && launches % 2) launches++;
         if (launches < sweeps) return relax_tiles(v, level, sweeps, launches, from);
     }
     const std::vector<int>& off = v.ops[level]->off;
     const bool centre_first = off[0] == 0 && off[1] == 0 && off[2] == 0;
-    if (v.relax_method != 2 || sweeps < 0 || !centre_first || (from == phi && sweeps % 2))
+    if (v.relax_method != 2 || sweeps < 0 || !centre_first ||
+        (from == phi && (sweeps % 2 || !other)))
         return gpd_operator_relax(v.ops[level], GPD_F64, v.relax_method, 1, phi, v.rhos[level],
                                   sweeps, v.weights[level], v.st);
-    return fd_jacobi_sweeps<double>(v.ops[level], 1, &from,
-                                    from == phi ? v.residuals[level] : phi, v.rhos[level], sweeps,
-                                    v.weights[level], v.st);
+    return fd_jacobi_sweeps<double>(v.ops[level], 1, &from, from == phi ? other : phi,
+                                    v.rhos[level], sweeps, v.weights[level], v.st);
 }
 
 // The first relaxation of a level below 0, where phi starts from zero
 static int relax_zero(const VCycle& v, int level, int sweeps)
 {
-    if (sweeps > 0 && sweeps_per_launch(v, level))
-        return relax_tiles(v, level, sweeps, relax_launches(v, level, sweeps), nullptr);
+    if (sweeps > 0 && sweeps_per_launch(v, level)) {
+        const int launches = relax_launches(v, level, sweeps);
+        if (launches == 1 || second_array(v, level))
+            return relax_tiles(v, level, sweeps, launches, nullptr);
+    }
     const long n = grid_points(v.ops[level]);
     hipLaunchKernelGGL(fill_zero_f64_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, v.st,
                        v.phis[level], n);
@@ -503,7 +513,6 @@ static int relax_zero(const VCycle& v, int level, int sweeps)
 // level 0; the level-0 residual and its norm are the caller's
 static int vcycle_level(const VCycle& v, int level)
 {
-    gpd_operator* op = v.ops[level];
     double* phi = v.phis[level];
     double* res = v.residuals[level];
     const int post = v.postsmooths[level];
@@ -547,8 +556,10 @@ extern "C" int gpd_poisson_vcycle(int levels, gpd_operator* const* ops,
     for (int l = 0; l <= levels; l++) {
         GPD_REQUIRE(ops[l] && phis[l] && rhos[l] && residuals[l], GPD_ERR_ARG,
                     "null operator or grid");
-        GPD_REQUIRE(phis[l] != rhos[l] && phis[l] != residuals[l], GPD_ERR_ARG,
-                    "phi, rho and residual must be distinct");
+        GPD_REQUIRE(phis[l] != rhos[l], GPD_ERR_ARG, "phi and rho must be distinct");
+        if (l < levels || l == 0)
+            GPD_REQUIRE(residuals[l] != phis[l] && residuals[l] != rhos[l], GPD_ERR_ARG,
+                        "phi, rho and residual must be distinct");
         if (l < levels) {
             GPD_REQUIRE(restrictors[l] && interpolators[l], GPD_ERR_ARG, "null transformer");
             GPD_REQUIRE(residuals[l] != rhos[l + 1] && phis[l + 1] != residuals[l] &&

@@ -291,8 +291,9 @@ class FDPoissonSolver:
         returns sum(residual^2) dv.  From level 0 the whole cycle is one
         library call (gpd_poisson_vcycle), which walks the levels with the
         differences formed in the stencils and the interpolations and the
-        coarsest levels in one launch; the grids are those of
-        iterate2_calls bit for bit."""
+        coarsest levels in one launch.  phi and the residual of level 0 and
+        the norm are those of iterate2_calls bit for bit; the grids below
+        are its scratch (some are not written at all)."""
         if level == 0:
             return self._vcycle()
         return self.iterate2_calls(step, level)

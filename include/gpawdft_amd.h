@@ -137,11 +137,14 @@ int gpd_transformer_destroy(gpd_transformer* t);
  * reference issues these calls one at a time from Python; here one call
  * walks the levels, so the host keeps ahead of the GPU.  The differences
  * are formed in the stencil and in the interpolation, and the coarsest
- * levels run in one launch where they fit a workgroup's LDS; every grid
- * gets the bits of the single calls.  A level's phi, rho and residual, its
+ * levels run in one launch where they fit a workgroup's LDS.  phi of level 0,
+ * its residual and the norm get the bits of the single calls; the other
+ * levels' grids are scratch: those inside the launch of the coarsest levels
+ * are not written but for the first one's phi, and a level's sweeps alternate
+ * between its phi and its residual.  A level's phi, rho and residual, its
  * residual and the next level's rho and phi, and the phi of consecutive
- * levels must be distinct.  Allocates only the stream-ordered temporaries
- * of relax and the dot. */
+ * levels must be distinct; below level 0 the coarsest level's residual is not
+ * used.  Allocates only the stream-ordered temporaries of relax and the dot. */
 int gpd_poisson_vcycle(int levels, gpd_operator* const* ops,
                        gpd_transformer* const* restrictors,
                        gpd_transformer* const* interpolators,
