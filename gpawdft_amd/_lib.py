@@ -109,7 +109,6 @@ _SIGNATURES = {
                                         _vp, _vp, _vp]),
     'gpd_leaky_relu': (_i, [_l, _f, _vp, _vp, _vp]),
     'gpd_leaky_relu_backward': (_i, [_l, _f, _vp, _vp, _vp, _vp]),
-    'gpd_scale_add': (_i, [_l, _f, _vp, _f, _vp, _vp]),
     'gpd_adam_step': (_i, [_l, _f, _f, _f, _f, _vp, _vp, _vp, _vp, _vp]),
 }
 

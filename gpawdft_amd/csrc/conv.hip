@@ -694,14 +694,6 @@ __global__ void leaky_relu_grad_kernel(long n, float a, const float* __restrict_
     if (i < n) gx[i] = x[i] > 0.f ? gy[i] : a * gy[i];
 }
 
-// y = alpha x + beta y, elementwise
-__global__ void scale_add_kernel(long n, float alpha, const float* __restrict__ x, float beta,
-                                 float* __restrict__ y)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) y[i] = alpha * x[i] + beta * y[i];
-}
-
 // Adam step on n parameters (bias-corrected learning rate lr_t)
 __global__ void adam_kernel(long n, float lr_t, float b1, float b2, float eps,
                             float* __restrict__ w, const float* __restrict__ g,
@@ -819,16 +811,6 @@ extern "C" int gpd_adam_step(long n, float lr_t, float beta1, float beta2, float
     if (n == 0) return GPD_OK;
     hipLaunchKernelGGL(adam_kernel, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, n,
                        lr_t, beta1, beta2, eps, d_w, d_g, d_m, d_v);
-    return last_error_to_status(hipGetLastError());
-}
-
-extern "C" int gpd_scale_add(long n, float alpha, const float* d_x, float beta, float* d_y,
-                             void* stream)
-{
-    GPD_REQUIRE(n >= 0 && (n == 0 || (d_x && d_y)), GPD_ERR_ARG, "bad arrays");
-    if (n == 0) return GPD_OK;
-    hipLaunchKernelGGL(scale_add_kernel, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream,
-                       n, alpha, d_x, beta, d_y);
     return last_error_to_status(hipGetLastError());
 }
 

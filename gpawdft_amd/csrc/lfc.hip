@@ -491,7 +491,6 @@ __global__ __launch_bounds__(64 * (P + Q)) void lfc_integrate_exact_kernel(
     constexpr int NB = NBL * Q;                // bands per workgroup
     constexpr int NP = kZ ? 2 : 1;             // parts of a value
     constexpr int BT = 8;                      // points per batch of LDS reads
-    constexpr int RB = 2;                      // batches of reads in registers
     __shared__ __attribute__((aligned(16))) double xs[3][NP][NB][CHP];
     __shared__ __attribute__((aligned(16))) double As[3][NFT][CHP];
 

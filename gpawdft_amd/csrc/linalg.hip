@@ -746,8 +746,7 @@ __global__ __launch_bounds__(kJT) void jacobi_small_kernel(T* __restrict__ A, in
 }
 
 // 16 x 16 block (w / 4, w % 4) of a 64 x 64 product by wave w: P Q, or P^H Q
-// (CT), on v_mfma_f64_16x16x4 (D: row 4 v + lane / 16, column lane % 16);
-// k < kend
+// (CT), on v_mfma_f64_16x16x4 (D: row 4 v + lane / 16, column lane % 16)
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 template <bool CT>
 __device__ __forceinline__ void wave_product(const double (&P)[kJB][kJB + 1],

@@ -246,8 +246,8 @@ class NewLocalizedFunctionsCollection:
     def set_launch(self, exact_bands):
         """Launch shape of the exact (FP64, complex) projections: 16, 32 or
         64 (the more, the more bands a workgroup takes), or 0 for the
-        automatic choice by the number of chains;
-        results do not depend on it."""
+        automatic choice by the number of workgroups; results do not depend
+        on it."""
         if exact_bands not in (0, 16, 32, 64):
             raise ValueError('exact_bands must be 0, 16, 32 or 64')
         self.exact_bands = int(exact_bands)

@@ -218,8 +218,9 @@ int gpd_lfc_set_phases(gpd_lfc* lfc, const double* phase_W);
 
 /* Launch knob of the exact (FP64, complex) integrate: 16, 32 or 64 (the
  * more, the more bands a workgroup takes), or 0 for the automatic choice,
- * which goes by the number of chains.  Results do not depend on it.  No counterpart in the reference (a tuning parameter of this
- * library's kernels).                                                  */
+ * which goes by the number of workgroups.  Results do not depend on it.  No
+ * counterpart in the reference (a tuning parameter of this library's
+ * kernels).                                                            */
 int gpd_lfc_set_launch(gpd_lfc* lfc, int exact_bands);
 
 int gpd_lfc_destroy(gpd_lfc* lfc);
@@ -462,11 +463,9 @@ int gpd_conv3d_backward_weight(int B, int Cin, int Cout, int D, int H, int W,
                                float* d_gw, float* d_gb, void* stream);
 int gpd_leaky_relu(long n, float slope, const float* d_x, float* d_y,
                    void* stream);
+/* Apart from a convolution or a transfer (UNet takes it in their epilogues). */
 int gpd_leaky_relu_backward(long n, float slope, const float* d_x,
                             const float* d_gy, float* d_gx, void* stream);
-/* y = alpha x + beta y */
-int gpd_scale_add(long n, float alpha, const float* d_x, float beta,
-                  float* d_y, void* stream);
 /* Adam: m = b1 m + (1-b1) g; v = b2 v + (1-b2) g^2; w -= lr_t m/(sqrt v+eps) */
 int gpd_adam_step(long n, float lr_t, float beta1, float beta2, float eps,
                   float* d_w, const float* d_g, float* d_m, float* d_v,
