@@ -314,10 +314,9 @@ def subspace_step(steps):
     """The mixed-precision subspace step at 112^3 x 512 (64 atoms): FP32
     bands; S = dv psi psi^T and H = dv psi (H psi)^T on split-bfloat16 MFMA
     (six bf16 products per useful one, FP32 then FP64 accumulation), the
-    FP64 inverse Cholesky and eigensolve, and the FP32 band rotation on
-    FP32 MFMA.  MFMA utilisation counts the issued bf16 products (6 per
-    useful multiply-add) against the dense bf16 peak, and the rotation's
-    against the FP32 matrix peak."""
+    FP64 inverse Cholesky and eigensolve, and the FP32 band rotation on the
+    same split products.  MFMA utilisation counts the issued bf16 products
+    (6 per multiply-add formed) against the dense bf16 peak."""
     import numpy as np
     import torch
     from gpawdft_amd import hs_operators as hs
@@ -363,14 +362,14 @@ def subspace_step(steps):
            'total_ms': sum(t.values()),
            'S_useful_tflops': useful_S / (t['S'] * 1e-3) / 1e12,
            'H_useful_tflops': useful_H / (t['H'] * 1e-3) / 1e12,
-           # the kernel computes both triangles: Nb^2 K MACs for S and H
-           'S_mfma_util_bf16': issued(Nb * Nb * K) / (t['S'] * 1e-3) /
-           2.5e15,
+           # S: the 128 x 128 tiles on and below the diagonal; H: all
+           'S_mfma_util_bf16': issued((Nb // 128) * (Nb // 128 + 1) // 2 *
+                                      128**2 * K) / (t['S'] * 1e-3) / 2.5e15,
            'H_mfma_util_bf16': issued(Nb * Nb * K) / (t['H'] * 1e-3) /
            2.5e15,
            'rotate_tflops': 2 * Nb * Nb * K / (t['rotate'] * 1e-3) / 1e12,
-           'rotate_mfma_util_f32': 2 * Nb * Nb * K / (t['rotate'] * 1e-3) /
-           157.3e12,
+           'rotate_mfma_util_bf16': issued(Nb * Nb * K) /
+           (t['rotate'] * 1e-3) / 2.5e15,
            'inverse_cholesky_gflops': Nb**3 / 3 / (t['inverse_cholesky'] *
                                                    1e-3) / 1e9}
     del psi, hpsi, out
