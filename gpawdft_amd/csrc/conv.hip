@@ -475,13 +475,13 @@ static int launch_conv(const ConvDims& d, const float* x, const float* w, const 
 // them, and the next pass's results follow the weights.
 //
 // A thread carries a chain (workgroup: a chunk) of 9 taps, one dz, of OB outputs
-// and IB inputs: 72 chains in registers fed by 9 IB + OB loads, of which the
-// next point's are in flight.  A channel's base is uniform, so that a point
+// and IB inputs: 72 chains in registers (OB = 8) fed by 9 IB + OB loads, of which
+// the next point's are in flight.  A channel's base is uniform, so that a point
 // costs 33 instructions of index arithmetic for its 72 FMAs.  Bound by the
 // vector units and the loads' way through the L1 in about equal parts, three
 // workgroups a CU (two with 16 outputs a thread: no gain).  Batch 8: 64^3 2 ->
-// 16 130 us and 16 -> 1 167, 32^3 16 -> 32 217, 32 -> 16 212, 16^3 32 -> 64 and
-// 64 -> 32 120.  A workgroup a pair of channels took 609, 333, 1134, 1127, 637
+// 16 128 us and 16 -> 1 178, 32^3 16 -> 32 217, 32 -> 16 212, 16^3 32 -> 64 and
+// 64 -> 32 119.  A workgroup a pair of channels took 609, 333, 1134, 1127, 637
 // and 633; products on the matrix units, in another order, 126, 85, 106, 108, 69
 // and 65.
 
@@ -632,8 +632,9 @@ __global__ __launch_bounds__(64) void wgrad_reduce_kernel(const float* __restric
     else gb[k - n] = s;
 }
 
-// A block of outputs by one input; for one or two outputs one of them by a
-// block of inputs.
+// A block of outputs by one input; for one or two outputs one of them by four
+// inputs (by eight, 64^3 16 -> 1 took 169 us, but one sample of 16^3, with six
+// workgroups, 36 with its launches, 24 now).
 static int launch_wgrad(const ConvDims& c, const float* x, const float* gy, float* gw, float* gb,
                         hipStream_t st)
 {
@@ -663,7 +664,7 @@ static int launch_wgrad(const ConvDims& c, const float* x, const float* gy, floa
     };
     const bool fits = 4 * npts * std::max(c.Cin, c.Cout) < (1L << 32);
     if (c.Cout <= 2)
-        fits ? launch(wgrad_kernel<1, 8, unsigned>, 1, 8) : launch(wgrad_kernel<1, 8, size_t>, 1, 8);
+        fits ? launch(wgrad_kernel<1, 4, unsigned>, 1, 4) : launch(wgrad_kernel<1, 4, size_t>, 1, 4);
     else
         fits ? launch(wgrad_kernel<8, 1, unsigned>, 8, 1) : launch(wgrad_kernel<8, 1, size_t>, 8, 1);
     int rc = last_error_to_status(hipGetLastError());
