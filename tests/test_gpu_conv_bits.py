@@ -146,3 +146,36 @@ def test_weight_gradient_keeps_its_order(cuda, B, Cin, Cout, shape):
     rgw, rgb = _wgrad(x, gy)
     assert np.array_equal(gw.cpu().numpy(), rgw)
     assert np.array_equal(gb.cpu().numpy(), rgb)
+
+
+@pytest.mark.parametrize('Cout', [1, 3])
+def test_weight_gradient_of_arrays_above_4_gib(cuda, Cout):
+    """Values at the end of a grid of 2^30 points, against the same values in
+    a small grid: all other products are zero.  At most 36 products a sum."""
+    import torch
+    import unet as U
+    from gpawdft_amd._lib import check, lib
+    from gpawdft_amd.device import stream_ptr
+    shape, small = (16, 8192, 8192), (6, 16, 16)
+    rng = np.random.default_rng(Cout)
+    x = np.zeros((1, 1) + small, np.float32)
+    x[..., -2:, -8:, -8:] = rng.standard_normal((2, 8, 8))
+    gy = np.zeros((1, Cout) + small, np.float32)
+    gy[..., -1:, -6:, -6:] = rng.standard_normal((1, Cout, 1, 6, 6))
+
+    def large(a):
+        t = torch.zeros(a.shape[:2] + shape, device='cuda')
+        t[..., -6:, -16:, -16:] = torch.from_numpy(a).cuda()
+        return t
+
+    dx, dgy = large(x), large(gy)
+    gw = torch.empty((Cout, 1, 27), dtype=torch.float32, device='cuda')
+    gb = torch.empty(Cout, dtype=torch.float32, device='cuda')
+    check(lib().gpd_conv3d_backward_weight(
+        1, 1, Cout, *shape, dx.data_ptr(), dgy.data_ptr(), gw.data_ptr(),
+        gb.data_ptr(), stream_ptr()))
+    rgw, rgb = U.conv3d_backward_weight(x.astype(float), gy.astype(float))
+    tol = 36 * 2.0**-24 * np.abs(gy).sum(axis=(0, 2, 3, 4)).max() * 4
+    assert np.abs(gw.cpu().numpy() - rgw).max() < tol
+    assert np.abs(gb.cpu().numpy() - rgb).max() < tol
+    assert np.abs(rgw).max() > 1000 * tol
